@@ -293,6 +293,15 @@ hipError_t fdr_fwd_h_segmented(const void* k, const void* w, const void* u, cons
                                void* workspace, hipStream_t stream);
 
 /*
+ * fdr_fwd_h_segmented (segments > 1) or fdr_fwd_h (segments = 1, workspace null) with v_new in the state's
+ * update as bf16 hi + lo instead of rounded to bf16 once; h and v_new are stored as those do.
+ */
+hipError_t fdr_fwd_h_split(const void* k, const void* w, const void* u, const float* g, int gate_mode,
+                           const float* h0, void* h, void* v_new, float* ht, int state_v_first, int B, int T,
+                           int H, int k_heads, int K, int V, int chunk, int segments, int value_block,
+                           void* workspace, hipStream_t stream);
+
+/*
  * fdr_fwd_h over a variable-length batch, with the packing, chunk_offsets and cu_seqlens of
  * fdr_state_bwd_varlen; h0 / ht per sequence [N,H,K,V].  Replaces FLA's
  * chunk_gated_delta_rule_fwd_h with cu_seqlens (the recompute policy's call).
@@ -534,6 +543,18 @@ hipError_t fdr_forward_scan(const void* q, const void* k, const void* v, const v
                             const int* chunk_offsets, const int* cu_seqlens, const int* chunk_indices, int B, int T,
                             int N, int H, int qk_heads, int K, int V, int chunk, float scale, int value_block, int segments, void* workspace,
                             hipStream_t stream);
+
+/* fdr_forward_scan of dense rows with v_new in the state's update as bf16 hi + lo (as fdr_fwd_h_split). */
+hipError_t fdr_forward_scan_split(const void* q, const void* k, const void* v, const void* g, int gate_mode,
+                                  int raw_gate, const float* A_log, const float* dt_bias, int has_lower_bound,
+                                  float lower_bound, const void* beta, const void* b_gate, const void* w_gate,
+                                  float norm_eps, int raw_beta, float beta_scale, void* q_norm, void* k_norm,
+                                  float* q_rnorm, float* k_rnorm, float* beta_out, float* gc, float* Aqk,
+                                  float* Akk, void* operands, const float* h0, void* o, float* ht,
+                                  int state_v_first, const int* chunk_offsets, const int* cu_seqlens,
+                                  const int* chunk_indices, int B, int T, int N, int H, int qk_heads, int K,
+                                  int V, int chunk, float scale, int value_block, int segments, void* workspace,
+                                  hipStream_t stream);
 
 /*
  * KDA's in-kernel gate activation (use_gate_in_kernel=True) and its backward, as the

@@ -31,6 +31,7 @@ SIGNATURES = {
     "fdr_state_bwd_varlen": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F,
                              _I, _P],
     "fdr_fwd_h_segmented": [_P, _P, _P, _P, _I, _P, _P, _P, _P] + [_I] * 10 + [_P, _P],
+    "fdr_fwd_h_split": [_P, _P, _P, _P, _I, _P, _P, _P, _P] + [_I] * 10 + [_P, _P],
     "fdr_fwd_h_varlen": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
     "fdr_fwd_h_wy": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I,
                      _I, _P],
@@ -55,6 +56,8 @@ SIGNATURES = {
                                      _P, _P, _I, _I, _I, _I, _I, _F, _P],
     "fdr_fwd_prepare_scan": [_P] * 4 + [_I, _I, _P, _P, _I, _F] + [_P] * 3 + [_F, _I, _F] + [_P] * 11 + [_I] * 7 + [_F, _P],
     "fdr_forward_scan": [_P] * 4 + [_I, _I, _P, _P, _I, _F] + [_P] * 3 + [_F, _I, _F] + [_P] * 12 + [_I] + [_P] * 3
+    + [_I] * 8 + [_F, _I, _I, _P, _P],
+    "fdr_forward_scan_split": [_P] * 4 + [_I, _I, _P, _P, _I, _F] + [_P] * 3 + [_F, _I, _F] + [_P] * 12 + [_I] + [_P] * 3
     + [_I] * 8 + [_F, _I, _I, _P, _P],
     "fdr_scalar_bwd_affine": [_P] * 4 + [_I] + [_P] * 12 + [ctypes.c_size_t, _F] + [_I] * 7 + [_F, _I, _P],
     "fdr_fwd_scan_o": [_P, _I, _P, _P, _P, _I, _P, _P] + [_I] * 6 + [_F, _I, _I, _P, _P],

@@ -12,6 +12,13 @@
 //   h       = diag(lambda_c) h + kg_c^T v_new_c
 //
 // h_c and v_new_c never leave the chip.
+//
+// SPLIT: v_new enters the state's update as bf16 hi + lo (16-bit mantissa) instead of one bf16, the precision
+// of the affine-step form, whose kg^T u goes into the state in fp32 (affine.hip).  It serves the calls that
+// form would take (few heads).  Final state against fp64, one bf16 / hi + lo / affine-step: DeltaNet B=1
+// T=2048 H=4 3.77e-3 / 3.11e-3 / 3.30e-3, KDA 3.26e-3 / 2.83e-3 / 2.83e-3; whole forward, us, one bf16 / hi + lo:
+// 45.8 / 47.9 and 55.4 / 58.7, KDA T=65536 H=16 1403 / 1473.  Of a segment's map only Q takes the split (P's
+// columns too: 1516 us, the same errors).
 #include "rewy_amd.h"
 
 #include "scan_body.hpp"
@@ -19,13 +26,14 @@
 
 namespace rewy {
 
-template <int BV>
+template <int BV, bool SPLIT>
 struct ScanOSmem {
   static constexpr int LDK = KD + 8;
   static constexpr int LDT = C + 8;
   bf16 k[2][C * KD];              // kg tile by chunk parity: read after a step's last barrier
   bf16 hT[BV][LDK];               // h^T
   bf16 vT[BV][LDT];               // v_new^T
+  bf16 vlT[SPLIT ? BV : 1][LDT];  // and its rest
 };
 
 // Eight waves own 16 state rows each; beside that waves 0-3 form v_new and waves 4-7 o, each for one
@@ -37,14 +45,14 @@ struct ScanOSmem {
 // against 338; GDN2 B=2 T=8192 H=32 253 (32-wide) against 432; KDA B=1 T=8192 H=32 196 (16-wide)
 // against 299, H=8 142 against 159.  All operands staged through LDS instead took 260, 396 and 314
 // (first, third and fourth); two chunks of prefetch instead of one 206, 265 and 207.
-template <int BV, bool VEC, bool MAP>
+template <int BV, bool VEC, bool MAP, bool SPLIT>
 __global__ __launch_bounds__(512) void fwd_scan_o_kernel(const char* __restrict__ ops, const float* __restrict__ h0,
                                                          bf16* __restrict__ o_out, float* __restrict__ ht_out, int T,
                                                          int H, float scale, const int* __restrict__ chunk_off,
                                                          int vf, const int* __restrict__ cu, int N, int segs,
                                                          const float* __restrict__ xseg,
                                                          const float* __restrict__ xlast) {
-  using S = ScanOSmem<BV>;
+  using S = ScanOSmem<BV, SPLIT>;
   __shared__ __attribute__((aligned(16))) S sm;
   constexpr int NVT = VD / BV;
   constexpr int NCT = BV / 16;
@@ -127,6 +135,10 @@ __global__ __launch_bounds__(512) void fwd_scan_o_kernel(const char* __restrict_
       f32x4 a = st[ct] * lam;
       a = mfma(k0, frag(&sm.vT[16 * ct][0], S::LDT), a);
       a = mfma(k1, frag(&sm.vT[16 * ct][32], S::LDT), a);
+      if constexpr (SPLIT) {
+        a = mfma(k0, frag(&sm.vlT[16 * ct][0], S::LDT), a);
+        a = mfma(k1, frag(&sm.vlT[16 * ct][32], S::LDT), a);
+      }
       st[ct] = a;
     }
   };
@@ -178,10 +190,10 @@ __global__ __launch_bounds__(512) void fwd_scan_o_kernel(const char* __restrict_
         for (int ct = 0; ct < NCT; ++ct) a[ct] = mfma(wf[ks], frag(&sm.hT[16 * ct][32 * ks], S::LDK), a[ct]);
 #pragma unroll
       for (int ct = 0; ct < NCT; ++ct) {
-        bf16x4 v4;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v4[r] = to_bf16(-a[ct][r]);
-        *reinterpret_cast<bf16x4*>(&sm.vT[16 * ct + lc][16 * drow + 4 * lg]) = v4;
+        bf16x4 lo;
+        const bf16x4 hi = split_hi4(-a[ct], lo);
+        *reinterpret_cast<bf16x4*>(&sm.vT[16 * ct + lc][16 * drow + 4 * lg]) = hi;
+        if constexpr (SPLIT) *reinterpret_cast<bf16x4*>(&sm.vlT[16 * ct + lc][16 * drow + 4 * lg]) = lo;
       }
       lds_barrier();
       update(db, lam);
@@ -287,17 +299,20 @@ __global__ __launch_bounds__(512) void fwd_scan_o_kernel(const char* __restrict_
 // image is copied.  P to pbuf [N (segs - 1), H, K, K], Q to qbuf likewise.  Bound by the step's chain as
 // the scan (2.1 us a chunk).  With the combine and the segments' scans (KDA, us, one scan / in segments):
 // H=16 1024 chunks 1434 / 705, 256 chunks 359 / 204, H=8 256 chunks 262 / 145, H=4 128 chunks 134 / 92.
+template <bool SPLIT>
 struct ScanXferSmem {
   static constexpr int LDK = KD + 8;
   static constexpr int LDT = C + 8;
   bf16 k[2][C * KD];       // by chunk parity
   bf16 hT[128][LDK];       // state^T: columns 0-63 of P's half, 64-127 of Q's
   bf16 vT[128][LDT];       // [-w P | u - w Q]^T
+  bf16 vlT[SPLIT ? 64 : 1][LDT];   // the rest of Q's columns
 };
 
+template <bool SPLIT>
 __global__ __launch_bounds__(512) void scan_xfer_kernel(const char* __restrict__ ops, float* __restrict__ pbuf,
                                                         float* __restrict__ qbuf, int T, int H, int segs) {
-  using S = ScanXferSmem;
+  using S = ScanXferSmem<SPLIT>;
   __shared__ __attribute__((aligned(16))) S sm;
   const int logical = xcd_logical_block();
   const int half = logical & 1;
@@ -376,10 +391,10 @@ __global__ __launch_bounds__(512) void scan_xfer_kernel(const char* __restrict__
         a[cc] = mfma(wf[ks], frag(&sm.hT[16 * (dct0 + cc)][32 * ks], S::LDK), a[cc]);
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc) {
-      bf16x4 v4;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v4[r] = to_bf16(-a[cc][r]);
-      *reinterpret_cast<bf16x4*>(&sm.vT[16 * (dct0 + cc) + lc][16 * drow + 4 * lg]) = v4;
+      bf16x4 lo;
+      const bf16x4 hi = split_hi4(-a[cc], lo);
+      *reinterpret_cast<bf16x4*>(&sm.vT[16 * (dct0 + cc) + lc][16 * drow + 4 * lg]) = hi;
+      if (SPLIT && q_half) *reinterpret_cast<bf16x4*>(&sm.vlT[16 * cc + lc][16 * drow + 4 * lg]) = lo;
     }
     lds_barrier();
     const bf16x8 k0 = frag_tr<16>(sm.k[db], 0, 16 * wv), k1 = frag_tr<16>(sm.k[db], 32, 16 * wv);
@@ -388,6 +403,12 @@ __global__ __launch_bounds__(512) void scan_xfer_kernel(const char* __restrict__
       f32x4 x = st[j] * lam;
       x = mfma(k0, frag(&sm.vT[16 * j][0], S::LDT), x);
       x = mfma(k1, frag(&sm.vT[16 * j][32], S::LDT), x);
+      if constexpr (SPLIT) {
+        if (j >= 4) {
+          x = mfma(k0, frag(&sm.vlT[16 * (j - 4)][0], S::LDT), x);
+          x = mfma(k1, frag(&sm.vlT[16 * (j - 4)][32], S::LDT), x);
+        }
+      }
       st[j] = x;
     }
     settle_chunk();
@@ -403,15 +424,15 @@ __global__ __launch_bounds__(512) void scan_xfer_kernel(const char* __restrict__
 
 template <int BV>
 static hipError_t launch_scan_o(const void* ops, bool vec, const float* h0, void* o, float* ht, int N, int T, int H,
-                                float scale, const int* co, int vf, const int* cu, int segs, float* ws,
+                                float scale, const int* co, int vf, const int* cu, int segs, float* ws, bool split,
                                 hipStream_t s) {
   const int grid = co ? packed_grid(N, H, VD / BV) : N * segs * H * (VD / BV);
   const float *xseg = nullptr, *xlast = nullptr;
   if (segs > 1) {
     const size_t maps = (size_t)N * (segs - 1) * H * KD * VD;
     float *pbuf = ws, *qbuf = ws + maps, *xb = ws + 2 * maps, *xl = ws + 3 * maps;
-    hipLaunchKernelGGL(scan_xfer_kernel, dim3(N * (segs - 1) * H * 2), dim3(512), 0, s, (const char*)ops, pbuf, qbuf, T,
-                       H, segs);
+    hipLaunchKernelGGL(split ? scan_xfer_kernel<true> : scan_xfer_kernel<false>, dim3(N * (segs - 1) * H * 2), dim3(512),
+                       0, s, (const char*)ops, pbuf, qbuf, T, H, segs);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(state_combine_kernel<false>, dim3(N * H, VD / COMB_COLS), dim3(256), 0, s, pbuf, qbuf, h0, xb, xl,
@@ -421,15 +442,18 @@ static hipError_t launch_scan_o(const void* ops, bool vec, const float* h0, void
     xseg = xb;
     xlast = xl;
   }
-#define SO_LAUNCH(VEC, MAP)                                                                                      \
-  hipLaunchKernelGGL((fwd_scan_o_kernel<BV, VEC, MAP>), dim3(grid), dim3(512), 0, s, (const char*)ops, h0, (bf16*)o, \
-                     ht, T, H, scale, co, vf, cu, N, segs, xseg, xlast)
-  if (vec) {
-    if (cu) SO_LAUNCH(true, true);
-    else SO_LAUNCH(true, false);
+#define SO_LAUNCH(VEC, MAP, SPLIT)                                                                              \
+  hipLaunchKernelGGL((fwd_scan_o_kernel<BV, VEC, MAP, SPLIT>), dim3(grid), dim3(512), 0, s, (const char*)ops, h0,   \
+                     (bf16*)o, ht, T, H, scale, co, vf, cu, N, segs, xseg, xlast)
+  if (split) {                                       // dense rows
+    if (vec) SO_LAUNCH(true, false, true);
+    else SO_LAUNCH(false, false, true);
+  } else if (vec) {
+    if (cu) SO_LAUNCH(true, true, false);
+    else SO_LAUNCH(true, false, false);
   } else {
-    if (cu) SO_LAUNCH(false, true);
-    else SO_LAUNCH(false, false);
+    if (cu) SO_LAUNCH(false, true, false);
+    else SO_LAUNCH(false, false, false);
   }
 #undef SO_LAUNCH
   return hipGetLastError();
@@ -453,17 +477,18 @@ extern "C" size_t fdr_scan_workspace_bytes(int N, int H, int segments) {
   return (size_t)N * H * (3 * (size_t)(segments - 1) + 1) * KD * VD * sizeof(float);
 }
 
-extern "C" hipError_t fdr_fwd_scan_o(const void* operands, int gate_mode, const float* h0, void* o, float* ht,
-                                     int state_v_first, const int* chunk_offsets, const int* cu_seqlens, int N,
-                                     int T, int H, int K, int V, int chunk, float scale, int value_block, int segments,
-                                     void* workspace, hipStream_t stream) {
+static hipError_t scan_o_dispatch(const void* operands, int gate_mode, const float* h0, void* o, float* ht,
+                                  int state_v_first, const int* chunk_offsets, const int* cu_seqlens, int N,
+                                  int T, int H, int K, int V, int chunk, float scale, int value_block, int segments,
+                                  void* workspace, bool split, hipStream_t stream) {
   if (K != KD || V != VD || chunk != C || T <= 0 || T % C || N <= 0 || H <= 0) return hipErrorInvalidValue;
   if (!operands || !o || gate_mode < RG_NONE || gate_mode > RG_VECTOR) return hipErrorInvalidValue;
   if (cu_seqlens && !chunk_offsets) return hipErrorInvalidValue;
+  if (split && chunk_offsets) return hipErrorInvalidValue;
   if (segments < 1 || segments > T / C || (segments > 1 && (chunk_offsets || !workspace))) return hipErrorInvalidValue;
   const int bv = value_block > 0 ? value_block : scan_o_bv(N * segments, H);
 #define SO_ARGS operands, gate_mode == RG_VECTOR, h0, o, ht, N, T, H, scale, chunk_offsets, state_v_first ? 1 : 0, \
-                cu_seqlens, segments, (float*)workspace, stream
+                cu_seqlens, segments, (float*)workspace, split, stream
   switch (bv) {
     case 16: return launch_scan_o<16>(SO_ARGS);
     case 32: return launch_scan_o<32>(SO_ARGS);
@@ -473,22 +498,30 @@ extern "C" hipError_t fdr_fwd_scan_o(const void* operands, int gate_mode, const 
 #undef SO_ARGS
 }
 
+extern "C" hipError_t fdr_fwd_scan_o(const void* operands, int gate_mode, const float* h0, void* o, float* ht,
+                                     int state_v_first, const int* chunk_offsets, const int* cu_seqlens, int N,
+                                     int T, int H, int K, int V, int chunk, float scale, int value_block, int segments,
+                                     void* workspace, hipStream_t stream) {
+  return scan_o_dispatch(operands, gate_mode, h0, o, ht, state_v_first, chunk_offsets, cu_seqlens, N, T, H, K, V, chunk,
+                         scale, value_block, segments, workspace, false, stream);
+}
+
 // The two launches as one host call: a short forward is bound by the host, and a foreign-function
 // call with its argument checks costs it ~8 us.
-extern "C" hipError_t fdr_forward_scan(const void* q, const void* k, const void* v, const void* g, int gate_mode,
-                                       int raw_gate, const float* A_log, const float* dt_bias, int has_lower_bound,
-                                       float lower_bound, const void* beta, const void* b_gate, const void* w_gate,
-                                       float norm_eps, int raw_beta, float beta_scale, void* q_norm, void* k_norm,
-                                       float* q_rnorm, float* k_rnorm, float* beta_out, float* gc, float* Aqk,
-                                       float* Akk, void* operands, const float* h0, void* o,
-                                       float* ht, int state_v_first, const int* chunk_offsets, const int* cu_seqlens,
-                                       const int* chunk_indices, int B, int T, int N, int H, int qk_heads, int K,
-                                       int V, int chunk, float scale, int value_block, int segments, void* workspace,
-                                       hipStream_t stream) {
+static hipError_t forward_scan_dispatch(const void* q, const void* k, const void* v, const void* g, int gate_mode,
+                                        int raw_gate, const float* A_log, const float* dt_bias, int has_lower_bound,
+                                        float lower_bound, const void* beta, const void* b_gate, const void* w_gate,
+                                        float norm_eps, int raw_beta, float beta_scale, void* q_norm, void* k_norm,
+                                        float* q_rnorm, float* k_rnorm, float* beta_out, float* gc, float* Aqk,
+                                        float* Akk, void* operands, const float* h0, void* o, float* ht,
+                                        int state_v_first, const int* chunk_offsets, const int* cu_seqlens,
+                                        const int* chunk_indices, int B, int T, int N, int H, int qk_heads, int K,
+                                        int V, int chunk, float scale, int value_block, int segments, void* workspace,
+                                        bool split, hipStream_t stream) {
   // what only fdr_fwd_scan_o would refuse, before the first launch (T here: as fdr_fwd_prepare_scan's)
   if (!o || N <= 0 || (!chunk_offsets && N != B) || (cu_seqlens && !chunk_offsets) || (chunk_offsets && B != 1) ||
       (value_block != 0 && value_block != 16 && value_block != 32 && value_block != 64) ||
-      segments < 1 || segments > T / C || (segments > 1 && (chunk_offsets || !workspace)))
+      segments < 1 || segments > T / C || (segments > 1 && (chunk_offsets || !workspace)) || (split && chunk_offsets))
     return hipErrorInvalidValue;
   const hipError_t st =
       fdr_fwd_prepare_scan(q, k, v, g, gate_mode, raw_gate, A_log, dt_bias, has_lower_bound, lower_bound, beta, b_gate,
@@ -496,6 +529,41 @@ extern "C" hipError_t fdr_forward_scan(const void* q, const void* k, const void*
                            Akk, operands, cu_seqlens, chunk_indices, B, T, H, qk_heads, K, V, chunk,
                            scale, stream);
   if (st != hipSuccess) return st;
-  return fdr_fwd_scan_o(operands, gate_mode, h0, o, ht, state_v_first, chunk_offsets, cu_seqlens, N, T, H, K, V, chunk,
-                        scale, value_block, segments, workspace, stream);
+  return scan_o_dispatch(operands, gate_mode, h0, o, ht, state_v_first, chunk_offsets, cu_seqlens, N, T, H, K, V, chunk,
+                         scale, value_block, segments, workspace, split, stream);
+}
+
+extern "C" hipError_t fdr_forward_scan(const void* q, const void* k, const void* v, const void* g, int gate_mode,
+                                       int raw_gate, const float* A_log, const float* dt_bias, int has_lower_bound,
+                                       float lower_bound, const void* beta, const void* b_gate, const void* w_gate,
+                                       float norm_eps, int raw_beta, float beta_scale, void* q_norm, void* k_norm,
+                                       float* q_rnorm, float* k_rnorm, float* beta_out, float* gc, float* Aqk,
+                                       float* Akk, void* operands, const float* h0, void* o, float* ht,
+                                       int state_v_first, const int* chunk_offsets, const int* cu_seqlens,
+                                       const int* chunk_indices, int B, int T, int N, int H, int qk_heads, int K,
+                                       int V, int chunk, float scale, int value_block, int segments, void* workspace,
+                                       hipStream_t stream) {
+  return forward_scan_dispatch(q, k, v, g, gate_mode, raw_gate, A_log, dt_bias, has_lower_bound, lower_bound, beta,
+                               b_gate, w_gate, norm_eps, raw_beta, beta_scale, q_norm, k_norm, q_rnorm, k_rnorm,
+                               beta_out, gc, Aqk, Akk, operands, h0, o, ht, state_v_first, chunk_offsets, cu_seqlens,
+                               chunk_indices, B, T, N, H, qk_heads, K, V, chunk, scale, value_block, segments,
+                               workspace, false, stream);
+}
+
+extern "C" hipError_t fdr_forward_scan_split(const void* q, const void* k, const void* v, const void* g, int gate_mode,
+                                             int raw_gate, const float* A_log, const float* dt_bias,
+                                             int has_lower_bound, float lower_bound, const void* beta,
+                                             const void* b_gate, const void* w_gate, float norm_eps, int raw_beta,
+                                             float beta_scale, void* q_norm, void* k_norm, float* q_rnorm,
+                                             float* k_rnorm, float* beta_out, float* gc, float* Aqk, float* Akk,
+                                             void* operands, const float* h0, void* o, float* ht, int state_v_first,
+                                             const int* chunk_offsets, const int* cu_seqlens, const int* chunk_indices,
+                                             int B, int T, int N, int H, int qk_heads, int K, int V, int chunk,
+                                             float scale, int value_block, int segments, void* workspace,
+                                             hipStream_t stream) {
+  return forward_scan_dispatch(q, k, v, g, gate_mode, raw_gate, A_log, dt_bias, has_lower_bound, lower_bound, beta,
+                               b_gate, w_gate, norm_eps, raw_beta, beta_scale, q_norm, k_norm, q_rnorm, k_rnorm,
+                               beta_out, gc, Aqk, Akk, operands, h0, o, ht, state_v_first, chunk_offsets, cu_seqlens,
+                               chunk_indices, B, T, N, H, qk_heads, K, V, chunk, scale, value_block, segments,
+                               workspace, true, stream);
 }

@@ -262,7 +262,9 @@ __global__ __launch_bounds__(256) void prepare_wu_kernel(
 // ------------------------------------------------------------------------------------------
 // fdr_fwd_h
 // ------------------------------------------------------------------------------------------
-template <int BV, int GATE>
+// SPLIT (fdr_fwd_h_split): v_new enters the state's update as bf16 hi + lo, why and where: fwd_scan.hip.
+// Saved KDA forward (us, one bf16 / hi + lo): B*H = 16 64 chunks 145 / 154, 1024 chunks 1725 / 1795.
+template <int BV, int GATE, bool SPLIT>
 struct FwdSmem {
   static constexpr int LDK = KD + 8;
   static constexpr int LDT = C + 8;
@@ -272,17 +274,18 @@ struct FwdSmem {
   bf16 k[2][C * KD];       // kg rows (swizzled): A operand of kg^T v_new (over T, transposed reads)
   bf16 hT[2][BV][LDK];     // h^T:    B operand of w h
   bf16 vT[BV][LDT];        // v_new^T: B operand of kg^T v_new
+  bf16 vlT[SPLIT ? BV : 1][LDT];   // and its rest
   bf16 u[C * BV];          // u rows [t][v] (swizzled): read transposed in the accumulator layout
   float lam[2][KD];
 };
 
-template <int BV, int GATE, bool MAP>
+template <int BV, int GATE, bool MAP, bool SPLIT>
 __global__ __launch_bounds__(512) void fwd_h_kernel(
     const bf16* __restrict__ k, const bf16* __restrict__ w, const bf16* __restrict__ u,
     const float* __restrict__ g, const float* __restrict__ h0, bf16* __restrict__ h_out,
     bf16* __restrict__ vnew_out, float* __restrict__ ht_out, int T, int H, const int* __restrict__ chunk_off,
     int vf, int HQ, const int* __restrict__ cu, int N, int segs) {
-  using S = FwdSmem<BV, GATE>;
+  using S = FwdSmem<BV, GATE, SPLIT>;
   __shared__ S sm;
   constexpr int NVT = VD / BV;
   constexpr int NCT = BV / 16;
@@ -444,10 +447,10 @@ __global__ __launch_bounds__(512) void fwd_h_kernel(
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
           a = mfma(frag(&sm.w[16 * drow][32 * ks], S::LDK), frag(&sm.hT[db][16 * ct][32 * ks], S::LDK), a);
-        bf16x4 v4;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v4[r] = to_bf16(-a[r]);
-        *reinterpret_cast<bf16x4*>(&sm.vT[16 * ct + (l & 15)][16 * drow + 4 * (l >> 4)]) = v4;
+        bf16x4 lo;
+        const bf16x4 hi = split_hi4(-a, lo);
+        *reinterpret_cast<bf16x4*>(&sm.vT[16 * ct + (l & 15)][16 * drow + 4 * (l >> 4)]) = hi;
+        if constexpr (SPLIT) *reinterpret_cast<bf16x4*>(&sm.vlT[16 * ct + (l & 15)][16 * drow + 4 * (l >> 4)]) = lo;
       }
     }
     lds_barrier();
@@ -460,6 +463,11 @@ __global__ __launch_bounds__(512) void fwd_h_kernel(
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
         a = mfma(frag_tr<16>(sm.k[db], 32 * ks, 16 * wv), frag(&sm.vT[16 * ct][32 * ks], S::LDT), a);
+      if constexpr (SPLIT) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          a = mfma(frag_tr<16>(sm.k[db], 32 * ks, 16 * wv), frag(&sm.vlT[16 * ct][32 * ks], S::LDT), a);
+      }
       st[ct] = a;
     }
     // stores of h_c and v_new_c from the transposed LDS copies (lanes run over rows)
@@ -507,6 +515,7 @@ __global__ __launch_bounds__(512) void fwd_h_kernel(
 // fwd_h_kernel's.  A scan of 1024 chunks at B*H = 16 is bound by its step chain with most CUs idle:
 // 1393 us direct and 1773 affine-step, against 624 in all for the maps, the chain and eight segments
 // of 128 (4 segments 965, 16 664).  P goes to pbuf [rows*segs, H, K, K], Q to qbuf [rows*segs, H, K, V].
+template <bool SPLIT>
 struct FwdXferSmem {
   static constexpr int LDK = KD + 8;
   static constexpr int LDT = C + 8;
@@ -514,15 +523,16 @@ struct FwdXferSmem {
   bf16 k[2][C * KD];       // per chunk parity, as lam (read after a step's last barrier)
   bf16 hT[128][LDK];       // state^T: columns 0-63 of P's half, 64-127 of Q's
   bf16 vT[128][LDT];       // [-w P | u - w Q]^T
+  bf16 vlT[SPLIT ? 64 : 1][LDT];   // the rest of Q's columns
   bf16 u[C * 64];          // the Q half's 64 value columns
   float lam[2][KD];
 };
 
-template <int GATE>
+template <int GATE, bool SPLIT>
 __global__ __launch_bounds__(512) void fwd_xfer_kernel(
     const bf16* __restrict__ k, const bf16* __restrict__ w, const bf16* __restrict__ u, const float* __restrict__ g,
     float* __restrict__ pbuf, float* __restrict__ qbuf, int T, int H, int HQ, int segs) {
-  using S = FwdXferSmem;
+  using S = FwdXferSmem<SPLIT>;
   __shared__ __attribute__((aligned(16))) S sm;
   constexpr int NTH = 512, CHV = 8;
   const int logical = xcd_logical_block();
@@ -619,10 +629,10 @@ __global__ __launch_bounds__(512) void fwd_xfer_kernel(
     }
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc) {
-      bf16x4 v4;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v4[r] = to_bf16(-a[cc][r]);
-      *reinterpret_cast<bf16x4*>(&sm.vT[16 * (dct0 + cc) + lc][16 * drow + 4 * lg]) = v4;
+      bf16x4 lo;
+      const bf16x4 hi = split_hi4(-a[cc], lo);
+      *reinterpret_cast<bf16x4*>(&sm.vT[16 * (dct0 + cc) + lc][16 * drow + 4 * lg]) = hi;
+      if (SPLIT && q_half) *reinterpret_cast<bf16x4*>(&sm.vlT[16 * cc + lc][16 * drow + 4 * lg]) = lo;
     }
     lds_barrier();
     const bf16x8 k0 = frag_tr<16>(sm.k[db], 0, 16 * wv), k1 = frag_tr<16>(sm.k[db], 32, 16 * wv);
@@ -632,6 +642,12 @@ __global__ __launch_bounds__(512) void fwd_xfer_kernel(
       f32x4 x = st[j] * lam;
       x = mfma(k0, frag(&sm.vT[16 * j][0], S::LDT), x);
       x = mfma(k1, frag(&sm.vT[16 * j][32], S::LDT), x);
+      if constexpr (SPLIT) {
+        if (j >= 4) {
+          x = mfma(k0, frag(&sm.vlT[16 * (j - 4)][0], S::LDT), x);
+          x = mfma(k1, frag(&sm.vlT[16 * (j - 4)][32], S::LDT), x);
+        }
+      }
       st[j] = x;
     }
     settle_chunk();
@@ -695,28 +711,36 @@ static hipError_t launch_prepare(const void* q, const void* k, const void* v, co
   return hipGetLastError();
 }
 
-template <int BV, int GATE>
+template <int BV, int GATE, bool SPLIT = false>
 static hipError_t launch_fwd_h(const void* k, const void* w, const void* u, const float* g, const float* h0,
                                void* h, void* vnew, float* ht, int B, int T, int H, hipStream_t s,
                                const int* co, int vf, int HQ, const int* cu, int segs = 0) {
   const int grid = co ? packed_grid(B, H, VD / BV) : B * (segs > 0 ? segs : 1) * H * (VD / BV);
 #define F_LAUNCH(MAP)                                                                                     \
-  hipLaunchKernelGGL((fwd_h_kernel<BV, GATE, MAP>), dim3(grid), dim3(512), 0, s, (const bf16*)k,          \
+  hipLaunchKernelGGL((fwd_h_kernel<BV, GATE, MAP, SPLIT>), dim3(grid), dim3(512), 0, s, (const bf16*)k,   \
                      (const bf16*)w, (const bf16*)u, g, h0, (bf16*)h, (bf16*)vnew, ht, T, H, co, vf, HQ, cu, B, segs)
-  if (cu) F_LAUNCH(true);
+  if constexpr (SPLIT) F_LAUNCH(false);     // (dense rows only)
+  else if (cu) F_LAUNCH(true);
   else F_LAUNCH(false);
 #undef F_LAUNCH
   return hipGetLastError();
 }
 
-template <int GATE>
+// segs = 1 with SPLIT: the direct scan
+template <int GATE, bool SPLIT>
 static hipError_t launch_fwd_segmented(const void* k, const void* w, const void* u, const float* g, const float* h0,
                                        void* h, void* vnew, float* ht, int B, int T, int H, int HQ, int segs, int bv,
                                        float* ws, int vf, hipStream_t s) {
+#define FS_SCAN(BV, H0, HT, VF, SEGS) \
+  launch_fwd_h<BV, GATE, SPLIT>(k, w, u, g, H0, h, vnew, HT, B, T, H, s, nullptr, VF, HQ, nullptr, SEGS)
+  if (SPLIT && segs == 1) {
+    if (bv == 16) return FS_SCAN(16, h0, ht, vf, 0);
+    return bv == 32 ? FS_SCAN(32, h0, ht, vf, 0) : FS_SCAN(64, h0, ht, vf, 0);
+  }
   const size_t n = (size_t)B * segs * H * KD * VD;
   float *pbuf = ws, *qbuf = ws + n, *xbuf = ws + 2 * n;
   // 1. per-segment maps
-  hipLaunchKernelGGL((fwd_xfer_kernel<GATE>), dim3(B * segs * H * 2), dim3(512), 0, s, (const bf16*)k, (const bf16*)w,
+  hipLaunchKernelGGL((fwd_xfer_kernel<GATE, SPLIT>), dim3(B * segs * H * 2), dim3(512), 0, s, (const bf16*)k, (const bf16*)w,
                      (const bf16*)u, g, pbuf, qbuf, T, H, HQ, segs);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -727,11 +751,12 @@ static hipError_t launch_fwd_segmented(const void* k, const void* w, const void*
   if (e != hipSuccess) return e;
   // 3. every segment from its start state (xbuf is [K,V] whatever the caller's state layout)
   switch (bv) {
-    case 16: return launch_fwd_h<16, GATE>(k, w, u, g, xbuf, h, vnew, nullptr, B, T, H, s, nullptr, 0, HQ, nullptr, segs);
-    case 32: return launch_fwd_h<32, GATE>(k, w, u, g, xbuf, h, vnew, nullptr, B, T, H, s, nullptr, 0, HQ, nullptr, segs);
-    case 64: return launch_fwd_h<64, GATE>(k, w, u, g, xbuf, h, vnew, nullptr, B, T, H, s, nullptr, 0, HQ, nullptr, segs);
+    case 16: return FS_SCAN(16, xbuf, nullptr, 0, segs);
+    case 32: return FS_SCAN(32, xbuf, nullptr, 0, segs);
+    case 64: return FS_SCAN(64, xbuf, nullptr, 0, segs);
     default: return hipErrorInvalidValue;
   }
+#undef FS_SCAN
 }
 
 }  // namespace rewy
@@ -864,12 +889,13 @@ extern "C" hipError_t fdr_fwd_h(const void* k, const void* w, const void* u, con
                         nullptr, state_v_first ? 1 : 0, nullptr);
 }
 
-extern "C" hipError_t fdr_fwd_h_segmented(const void* k, const void* w, const void* u, const float* g, int gate_mode,
+template <bool SPLIT>
+static hipError_t fwd_h_segmented_dispatch(const void* k, const void* w, const void* u, const float* g, int gate_mode,
                                           const float* h0, void* h, void* v_new, float* ht, int state_v_first, int B,
                                           int T, int H, int k_heads, int K, int V, int chunk, int segments,
                                           int value_block, void* workspace, hipStream_t stream) {
   if (K != KD || V != VD || chunk != C || T <= 0 || T % C || B <= 0 || H <= 0) return hipErrorInvalidValue;
-  if (!k || !w || !u || !h || !v_new || !workspace) return hipErrorInvalidValue;
+  if (!k || !w || !u || !h || !v_new || (!workspace && (!SPLIT || segments > 1))) return hipErrorInvalidValue;
   if (gate_mode != RG_NONE && !g) return hipErrorInvalidValue;
   if (segments < 1 || segments > T / C) return hipErrorInvalidValue;
   const int HQ = k_heads > 0 ? k_heads : H;
@@ -878,12 +904,28 @@ extern "C" hipError_t fdr_fwd_h_segmented(const void* k, const void* w, const vo
   if (bv != 16 && bv != 32 && bv != 64) return hipErrorInvalidValue;
 #define FS_ARGS k, w, u, g, h0, h, v_new, ht, B, T, H, HQ, segments, bv, (float*)workspace, state_v_first ? 1 : 0, stream
   switch (gate_mode) {
-    case RG_NONE: return launch_fwd_segmented<RG_NONE>(FS_ARGS);
-    case RG_SCALAR: return launch_fwd_segmented<RG_SCALAR>(FS_ARGS);
-    case RG_VECTOR: return launch_fwd_segmented<RG_VECTOR>(FS_ARGS);
+    case RG_NONE: return launch_fwd_segmented<RG_NONE, SPLIT>(FS_ARGS);
+    case RG_SCALAR: return launch_fwd_segmented<RG_SCALAR, SPLIT>(FS_ARGS);
+    case RG_VECTOR: return launch_fwd_segmented<RG_VECTOR, SPLIT>(FS_ARGS);
     default: return hipErrorInvalidValue;
   }
 #undef FS_ARGS
+}
+
+extern "C" hipError_t fdr_fwd_h_segmented(const void* k, const void* w, const void* u, const float* g, int gate_mode,
+                                          const float* h0, void* h, void* v_new, float* ht, int state_v_first, int B,
+                                          int T, int H, int k_heads, int K, int V, int chunk, int segments,
+                                          int value_block, void* workspace, hipStream_t stream) {
+  return fwd_h_segmented_dispatch<false>(k, w, u, g, gate_mode, h0, h, v_new, ht, state_v_first, B, T, H, k_heads, K, V,
+                                         chunk, segments, value_block, workspace, stream);
+}
+
+extern "C" hipError_t fdr_fwd_h_split(const void* k, const void* w, const void* u, const float* g, int gate_mode,
+                                      const float* h0, void* h, void* v_new, float* ht, int state_v_first, int B,
+                                      int T, int H, int k_heads, int K, int V, int chunk, int segments,
+                                      int value_block, void* workspace, hipStream_t stream) {
+  return fwd_h_segmented_dispatch<true>(k, w, u, g, gate_mode, h0, h, v_new, ht, state_v_first, B, T, H, k_heads, K, V,
+                                         chunk, segments, value_block, workspace, stream);
 }
 
 extern "C" hipError_t fdr_fwd_h_varlen(const void* k, const void* w, const void* u, const float* g, int gate_mode,

@@ -77,12 +77,14 @@ def chunk_forward_hip(op, q, k, v, g=None, beta=None, b=None, w=None, initial_st
     vec = gm == ops.GATE_VECTOR
     N, H = (B if varlen is None else varlen.N), v.shape[2]
     form = "auto" if varlen is None else "direct"
+    split = varlen is None and ops.split_pays(N, H, T // ops.CHUNK)
     if keep != "all" and varlen is None:
         form = _states_form(N, H, HQ, T // ops.CHUNK)
     if keep != "all" and (varlen is not None or form is None):
         o, final, saved = ops.forward_scan(q, k, v, g, gm, beta=beta, b=b, w=w, scale=scale, h0=h0,
                                            want_final=output_final_state, state_v_first=state_v_first, varlen=varlen,
-                                           gate=gate, want_saved=keep is not None, norm=norm, beta_act=beta_act)
+                                           gate=gate, want_saved=keep is not None, norm=norm, beta_act=beta_act,
+                                           split=split)
         saved["scale"] = scale
         return o, final, saved
     rq = rk = None
@@ -111,7 +113,7 @@ def chunk_forward_hip(op, q, k, v, g=None, beta=None, b=None, w=None, initial_st
                                               want_qg=vec and want_qg, gate=gate)
         h, v_new, final = ops.fwd_h(wu["kg"] if vec else k, wu["w"], wu["u"], gc, gm, h0=h0,
                                     want_final=output_final_state, varlen=varlen,
-                                    method=form, state_v_first=state_v_first)
+                                    method=form, state_v_first=state_v_first, split=split)
     o = ops.fwd_o(q, gc, gm, Aqk, h, v_new, scale, varlen=varlen)
     saved = dict(gc=gc, Aqk=Aqk, Akk=Akk, w=wu["w"], u=wu["u"], qg=wu["qg"], kg=wu["kg"], v_new=v_new, h=h,
                  scale=scale)
