@@ -159,3 +159,11 @@ def test_packed_work_group_order(lens, H):
                 assert torch.equal(x, y), (n, vb)
             a, c = a + m, c + nc
     torch.cuda.synchronize()
+
+
+def test_varlen_takes_device_offsets():
+    """cu_seqlens on the device, whole or as a list of scalars."""
+    from rewy_amd import ops
+    cu = torch.tensor([0, 64, 100], device="cuda")
+    for x in (cu, list(cu)):
+        assert ops.Varlen(x, cu.device).chunk_indices.tolist() == [[0, 0], [1, 0]]

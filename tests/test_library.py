@@ -319,6 +319,25 @@ def test_integration_guide_ctypes_lines_match_the_bindings():
     assert seen >= 10
 
 
+def test_varlen_takes_what_as_tensor_takes():
+    """Lists, tuples, arrays and lists of scalar tensors; not text, wrong shapes or falling offsets.  Not on a
+    default device either."""
+    import numpy as np
+    import torch
+    from rewy_amd import ops
+    for cu in ([0, 64, 100], (0, 64, 100), np.array([0, 64, 100], np.int32), torch.tensor([0, 64, 100]),
+               [torch.tensor(0), torch.tensor(64), torch.tensor(100)], [0.0, 64.0, 100.0]):
+        vl = ops.Varlen(cu, "cpu")
+        assert vl.cu_seqlens.tolist() == [0, 64, 100] and vl.chunk_offsets.tolist() == [0, 1, 2]
+        assert vl.chunk_indices.tolist() == [[0, 0], [1, 0]] and (vl.N, vl.T, vl.NC) == (2, 100, 2)
+    for bad in (["0", "64"], [[0, 64]], [0], [1, 64], [0, 64, 32], [0, 0]):
+        with pytest.raises((TypeError, ValueError)):
+            ops.Varlen(bad, "cpu")
+    cu = torch.tensor([0, 64, 100])
+    with torch.device("meta"):
+        assert ops.Varlen(cu, "cpu").chunk_indices.tolist() == [[0, 0], [1, 0]]
+
+
 def test_packed_tile_rules():
     """Tile widths of a packed batch's recurrences: the step chain of its longest sequence against all
     chunk steps spread over the CUs; the two recurrences on two streams only for long sequences, and
