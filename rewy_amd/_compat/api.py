@@ -69,7 +69,7 @@ class ChunkFunction(torch.autograd.Function):
         if backend == "optimized" and q.is_cuda:
             from ..hip_forward import chunk_forward_hip
             from ..ops import Varlen
-            varlen = None if cu_seqlens is None else Varlen(cu_seqlens, q.device)
+            varlen = None if cu_seqlens is None else Varlen(cu_seqlens, q.device, wait=False)
             ctx.cu_seqlens = varlen            # the chunk map, reused by the backward
             o, final, sv = chunk_forward_hip(op, q, k, v, g=g, beta=beta, b=b, w=w,
                                              initial_state=initial_state, scale=scale,

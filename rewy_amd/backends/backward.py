@@ -53,7 +53,7 @@ def _varlen(q, kw):
     B, T = q.shape[:2]
     if B != 1:
         raise ValueError(f"The batch size is expected to be 1 rather than {B} when using `cu_seqlens`.")
-    vl = cu if isinstance(cu, ops.Varlen) else ops.Varlen(cu, q.device)
+    vl = cu if isinstance(cu, ops.Varlen) else ops.Varlen(cu, q.device, wait=False)
     if vl.T != T:
         raise ValueError("cu_seqlens must rise from 0 to T")
     return vl

@@ -40,7 +40,7 @@ def varlen_of(q, cu_seqlens, chunk_indices, what):
         return None
     if q.shape[0] != 1:
         raise ValueError(f"The batch size is expected to be 1 rather than {q.shape[0]} when using `cu_seqlens`.")
-    vl = cu_seqlens if isinstance(cu_seqlens, ops.Varlen) else ops.Varlen(cu_seqlens, q.device)
+    vl = cu_seqlens if isinstance(cu_seqlens, ops.Varlen) else ops.Varlen(cu_seqlens, q.device, wait=False)
     if vl.T != q.shape[1]:
         raise ValueError("cu_seqlens must rise from 0 to T")
     if chunk_indices is not None and tuple(chunk_indices.shape) != (vl.NC, 2):

@@ -62,17 +62,36 @@ def test_affine_backward_call(op, vf, states, monkeypatch):
 
 
 def test_packed_tables_behind_other_work():
-    """The tables' copy waits for nothing and nothing overwrites its source before it ran: many batches
-    enqueued behind a long kernel each hold their own tables."""
+    """Without ``wait`` the tables' copy waits for nothing and nothing overwrites its source before it ran:
+    many batches enqueued behind a long kernel each hold their own tables."""
     from rewy_amd import ops
     dev = torch.device("cuda")
     x = torch.randn(4096, 4096, device=dev)
     for _ in range(20):
         x = x @ x * 1e-2
-    tables = [ops.Varlen([0, 10 + i, 200 + 3 * i], dev) for i in range(50)]
+    tables = [ops.Varlen([0, 10 + i, 200 + 3 * i], dev, wait=False) for i in range(50)]
     torch.cuda.synchronize()
     for i, t in enumerate(tables):
         cu = [0, 10 + i, 200 + 3 * i]
         nch = [-(-(b - a) // 64) for a, b in zip(cu, cu[1:])]
         assert t.cu_seqlens.tolist() == cu and t.chunk_offsets.tolist() == [0, nch[0], sum(nch)]
         assert t.chunk_indices.tolist() == [[n, j] for n, m in enumerate(nch) for j in range(m)]
+
+
+def test_packed_tables_are_ready_for_any_stream():
+    """A Varlen made behind a long kernel on one stream is read on another without a wait between them."""
+    from rewy_amd import ops
+    dev = torch.device("cuda")
+    side = torch.cuda.Stream()
+    cu = [0, 100, 164, 300]
+    want = [[0, 0], [0, 1], [1, 0], [2, 0], [2, 1], [2, 2]]
+    stale = torch.full((64,), -1, device=dev, dtype=torch.int32)     # what a table not yet copied would show
+    torch.cuda.synchronize()
+    del stale
+    torch.cuda._sleep(100_000_000)
+    vl = ops.Varlen(cu, dev)
+    with torch.cuda.stream(side):
+        got = [x.clone() for x in (vl.cu_seqlens, vl.chunk_offsets, vl.chunk_indices)]
+    side.synchronize()
+    assert got[0].tolist() == cu and got[1].tolist() == [0, 2, 3, 6] and got[2].tolist() == want
+    torch.cuda.synchronize()
