@@ -70,6 +70,8 @@ class ChunkFunction(torch.autograd.Function):
             from ..hip_forward import chunk_forward_hip
             from ..ops import Varlen
             varlen = None if cu_seqlens is None else Varlen(cu_seqlens, q.device, wait=False)
+            if norm:        # the raw rows that the forward reads are the ones saved: one copy of strided q / k
+                q, k = q.contiguous(), k.contiguous()
             ctx.cu_seqlens = varlen            # the chunk map, reused by the backward
             o, final, sv = chunk_forward_hip(op, q, k, v, g=g, beta=beta, b=b, w=w,
                                              initial_state=initial_state, scale=scale,
@@ -79,7 +81,7 @@ class ChunkFunction(torch.autograd.Function):
                                              gate=None if gate is None else (gate[0], A_log, dt_bias),
                                              norm=norm, beta_act=beta_act)
             if norm and grad:
-                raw_qk = (q.contiguous(), k.contiguous(), sv["rq"], sv["rk"])
+                raw_qk = (q, k, sv["rq"], sv["rk"])
                 q, k = sv["q"], sv["k"]
             if beta_act is not None:
                 beta = sv["beta"]

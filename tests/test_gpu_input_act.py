@@ -148,3 +148,35 @@ def test_norm_backward_refusals():
     with pytest.raises(ValueError):                       # the vector-gate families'
         ops.chunk_bwd(xs["q"], xs["k"], xs["v"], xs["v"], dO.cuda(), dO.cuda(), xs["g"], 1,
                       torch.zeros(1, 64, 2, 64, device="cuda"), z, z, 0.088, beta=xs["beta"], qk_rnorm=(r, r))
+
+
+@pytest.mark.parametrize("op,lens", [("kda", None), ("gdn", None), ("gdn", (65, 63))])
+def test_strided_rows_are_copied_once(op, lens, monkeypatch):
+    """q and k as slices of one projection: the contiguous copies that the forward reads are the ones saved for
+    the backward, and the result is the contiguous rows'."""
+    import rewy_amd as fdr
+    from rewy_amd import ops
+    xs, dO = make_inputs(op, 1, 128, 2, seed=19, h0=False)
+    xs = {n: x.cuda() for n, x in xs.items()}
+    qkv = torch.cat([xs[n] for n in ("q", "k", "v")], -1)
+    read, saved = [], []
+    real = ops.forward_scan
+    monkeypatch.setattr(ops, "forward_scan", lambda q, k, *a, **kw: (read.append((q, k)),      # (kept alive)
+                                                                      real(q, k, *a, **kw))[1])
+    kw = dict(use_qk_l2norm_in_kernel=True)
+    if lens:
+        kw["cu_seqlens"] = torch.tensor([0, *lens]).cumsum(0).cuda()
+
+    def run(q, k):
+        ys = [x.detach().requires_grad_() for x in (q, k)]
+        with fdr.use_backend("optimized"), torch.autograd.graph.saved_tensors_hooks(
+                lambda x: (saved.append(x.data_ptr()), x)[1], lambda x: x):
+            o, _ = {"kda": fdr.chunk_kda, "gdn": fdr.chunk_gated_delta_rule}[op](
+                *ys, xs["v"], xs["g"], xs["beta"], **kw)
+        return (o, *torch.autograd.grad(o, ys, dO.cuda()))
+    got = run(qkv[..., :128], qkv[..., 128:256])
+    assert len(read) == 1 and {x.data_ptr() for x in read[0]} <= set(saved)
+    want = run(xs["q"], xs["k"])
+    torch.cuda.synchronize()
+    for a, r in zip(got, want):
+        assert torch.equal(a, r)
