@@ -20,6 +20,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // structs whose copies lower to memcpy, which keeps them out of registers
 // (the backend then parks them in LDS or scratch).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// Two / four consecutive floats of a caller's fp32 tensor (gates, states, dt_bias), which may be a slice of a
+// flat buffer and start at any float.  Global memory takes such a load or store as one instruction all the same.
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float2 load2(const float* p) {
+  const f32x2u x = *reinterpret_cast<const f32x2u*>(p);
+  return {x[0], x[1]};
+}
 
 constexpr int C = 64;     // chunk length
 constexpr int KD = 128;   // key width

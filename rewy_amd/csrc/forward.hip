@@ -173,13 +173,13 @@ __global__ __launch_bounds__(512, 4) void fwd_prepare_kernel(
           rw.src(reinterpret_cast<const bf16*>(graw_) + kofs + (size_t)(8 * wv + r) * rsk + gcol, 8 * wv + r));
   }
   if constexpr (RAW != 0) {
-    if (act.dt_bias) gbias = *reinterpret_cast<const float2*>(act.dt_bias + h * KD + gcol);
+    if (act.dt_bias) gbias = load2(act.dt_bias + h * KD + gcol);
     if (act.A_log) ga_log = act.A_log[h];
   }
   if constexpr (VEC && RAW != 2) {
 #pragma unroll
     for (int r = 0; r < 8; ++r)
-      gv[r] = *reinterpret_cast<const float2*>(rw.src(graw + kofs + (size_t)(8 * wv + r) * rsk + gcol, 8 * wv + r));
+      gv[r] = load2(rw.src(graw + kofs + (size_t)(8 * wv + r) * rsk + gcol, 8 * wv + r));
   }
   float gx = 0.f;
   if constexpr (GATE == FG_SCALAR) gx = *rw.src(graw + (tok0 + l) * H + h, l);
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(512, 4) void fwd_prepare_kernel(
       const int t = 8 * wv + r;
       const float2 x = {(gv[r].x + carry.x) * fwd::RCP_LN2, (gv[r].y + carry.y) * fwd::RCP_LN2};
       *reinterpret_cast<float2*>(sg + gx_off(t, gcol)) = x;
-      if (!SOP || gc_out) *reinterpret_cast<float2*>(rw.dst(gc_out + kofs + (size_t)t * rsk + gcol, t)) = x;
+      if (!SOP || gc_out) *reinterpret_cast<f32x2u*>(rw.dst(gc_out + kofs + (size_t)t * rsk + gcol, t)) = f32x2u{x.x, x.y};
       if (SOP && t == C - 1)
         *reinterpret_cast<float2*>(sop + sop::LAM + 4 * gcol) = float2{fast_exp2(x.x), fast_exp2(x.y)};
     }

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(256) void state_combine_kernel(const float* __restr
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[e] = d[(col + e) * KD + r];
     } else {
-      x = *reinterpret_cast<const f32x4*>(d + r * VD + col);
+      x = *reinterpret_cast<const f32x4u*>(d + r * VD + col);
     }
   }
   f32x4 pre[KD * KD / 4 / 256];
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256) void state_combine_kernel(const float* __restr
 #pragma unroll
       for (int e = 0; e < 4; ++e) d[(col + e) * KD + r] = x[e];
     } else {
-      *reinterpret_cast<f32x4*>(d + r * VD + col) = x;
+      *reinterpret_cast<f32x4u*>(d + r * VD + col) = x;
     }
   }
 }

@@ -180,3 +180,36 @@ def test_strided_rows_are_copied_once(op, lens, monkeypatch):
     torch.cuda.synchronize()
     for a, r in zip(got, want):
         assert torch.equal(a, r)
+
+
+@pytest.mark.parametrize("NT,raw", [(3, False), (3, True), (96, False)])
+def test_fp32_inputs_start_at_any_float(NT, raw):
+    """Gate, dt_bias and initial state as slices of flat buffers that start one float in (96 chunks: the state
+    goes through the segments' chain): the aligned tensors' bits."""
+    import rewy_amd as fdr
+    from rewy_amd import ops
+    assert (ops.scan_segments(1, 2, NT) > 1) == (NT == 96)
+    xs, _ = make_inputs("kda", 1, 64 * NT, 2, seed=23, gate="mild")
+    xs = {n: x.cuda() for n, x in xs.items()}
+    kw = {}
+    if raw:
+        xs["g"] = _raw(xs["g"].cpu(), 3).float().cuda()
+        kw = dict(use_gate_in_kernel=True, A_log=torch.zeros(2, device="cuda"),
+                  dt_bias=torch.linspace(-1, 1, 256, device="cuda"))
+
+    def shifted(x):
+        flat = torch.empty(x.numel() + 1, device=x.device, dtype=x.dtype)
+        y = flat[1:].view(x.shape)
+        y.copy_(x)
+        assert y.is_contiguous() and y.data_ptr() % 8 == 4
+        return y
+
+    def run(f):
+        a = {n: f(x) if n in ("g", "initial_state") else x for n, x in xs.items()}
+        b = {n: f(x) if n == "dt_bias" else x for n, x in kw.items() if n != "use_gate_in_kernel"}
+        with fdr.use_backend("optimized"), torch.no_grad():
+            return fdr.chunk_kda(**a, **b, use_gate_in_kernel=raw, output_final_state=True)
+    got, want = run(shifted), run(lambda x: x)
+    torch.cuda.synchronize()
+    for a, r in zip(got, want):
+        assert torch.equal(a, r)
