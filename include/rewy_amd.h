@@ -285,7 +285,7 @@ hipError_t fdr_fwd_h(const void* k, const void* w, const void* u, const float* g
 /*
  * fdr_fwd_h with each row split into `segments` (1 .. T / 64) segments: their affine maps formed in
  * parallel, chained, and every segment run from its start state.  For long rows and few heads.
- * workspace: fdr_state_bwd_segmented_workspace_bytes(B, H, segments) bytes.
+ * workspace: fdr_state_bwd_segmented_workspace_bytes(B, H, segments) bytes, 16-byte aligned.
  */
 hipError_t fdr_fwd_h_segmented(const void* k, const void* w, const void* u, const float* g, int gate_mode,
                                const float* h0, void* h, void* v_new, float* ht, int state_v_first, int B, int T,
@@ -504,7 +504,7 @@ hipError_t fdr_fwd_o_varlen(const void* q, const float* gc, int gate_mode, const
  * The forward for a caller that keeps no states, in two launches.
  *
  * fdr_fwd_prepare_scan: fdr_fwd_prepare_wu, but w, u, kg, q 2^gc and Aqk go to `operands`
- * (fdr_scan_operands_bytes(number of chunks, H) bytes, 256-byte aligned) in the layout that
+ * (fdr_scan_operands_bytes(number of chunks, H) bytes, 16-byte aligned) in the layout that
  * fdr_fwd_scan_o reads.  gc, Aqk and Akk are also written as fdr_fwd_prepare writes them where
  * the pointer is not null.  norm_eps > 0: q and k are raw and L2-normalised on load as
  * fdr_l2norm_fwd does (q_norm, k_norm, q_rnorm, k_rnorm: its outputs for the backward, all or none).
@@ -516,7 +516,7 @@ hipError_t fdr_fwd_o_varlen(const void* q, const float* gc, int gate_mode, const
  * they start anywhere, as for fdr_fwd_h_varlen).  value_block 16, 32, 64, or 0 for the default.
  * segments > 1 (dense rows of at least as many chunks): each row in that many segments scanned side by
  * side, their start states from the segments' maps (as fdr_fwd_h_segmented); `workspace` then holds
- * fdr_scan_workspace_bytes(N, H, segments) bytes.
+ * fdr_scan_workspace_bytes(N, H, segments) bytes, 16-byte aligned.
  */
 size_t fdr_scan_operands_bytes(int num_chunks, int H);
 size_t fdr_scan_workspace_bytes(int N, int H, int segments);

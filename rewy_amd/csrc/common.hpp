@@ -111,6 +111,9 @@ __device__ __forceinline__ int packed_logical(const int* __restrict__ chunk_off,
   }
   return (n * H + pair % H) * NVT + vt;
 }
+// a buffer that the kernels read and write in 16-byte pieces
+inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
 inline int packed_grid(int N, int H, int NVT) { return (N * H + 7) / 8 * 8 * NVT; }
 
 // q / k may have fewer heads (HQ) than the value side (H): grouped value heads, FLA's head

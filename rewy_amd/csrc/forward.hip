@@ -961,6 +961,7 @@ extern "C" hipError_t fdr_fwd_prepare_scan(const void* q, const void* k, const v
   const InputAct in{norm_eps, (bf16*)q_norm, (bf16*)k_norm, q_rnorm, k_rnorm, raw_beta, beta_scale, beta_out};
   if (K != KD || V != VD || chunk != C || T <= 0 || T % C || B <= 0 || H <= 0 || !operands)
     return hipErrorInvalidValue;
+  if (!aligned16(operands)) return hipErrorInvalidValue;
   if ((cu_seqlens == nullptr) != (chunk_indices == nullptr) || (cu_seqlens && B != 1)) return hipErrorInvalidValue;
   const GateAct act{A_log, dt_bias, lower_bound, has_lower_bound ? (A_log ? 1 : 2) : 0};
   if (cu_seqlens)

@@ -485,6 +485,7 @@ static hipError_t scan_o_dispatch(const void* operands, int gate_mode, const flo
   if (!operands || !o || gate_mode < RG_NONE || gate_mode > RG_VECTOR) return hipErrorInvalidValue;
   if (cu_seqlens && !chunk_offsets) return hipErrorInvalidValue;
   if (split && chunk_offsets) return hipErrorInvalidValue;
+  if (!aligned16(operands) || !aligned16(workspace)) return hipErrorInvalidValue;
   if (segments < 1 || segments > T / C || (segments > 1 && (chunk_offsets || !workspace))) return hipErrorInvalidValue;
   const int bv = value_block > 0 ? value_block : scan_o_bv(N * segments, H);
 #define SO_ARGS operands, gate_mode == RG_VECTOR, h0, o, ht, N, T, H, scale, chunk_offsets, state_v_first ? 1 : 0, \
@@ -521,7 +522,8 @@ static hipError_t forward_scan_dispatch(const void* q, const void* k, const void
   // what only fdr_fwd_scan_o would refuse, before the first launch (T here: as fdr_fwd_prepare_scan's)
   if (!o || N <= 0 || (!chunk_offsets && N != B) || (cu_seqlens && !chunk_offsets) || (chunk_offsets && B != 1) ||
       (value_block != 0 && value_block != 16 && value_block != 32 && value_block != 64) ||
-      segments < 1 || segments > T / C || (segments > 1 && (chunk_offsets || !workspace)) || (split && chunk_offsets))
+      segments < 1 || segments > T / C || (segments > 1 && (chunk_offsets || !workspace)) || (split && chunk_offsets) ||
+      !aligned16(workspace))
     return hipErrorInvalidValue;
   const hipError_t st =
       fdr_fwd_prepare_scan(q, k, v, g, gate_mode, raw_gate, A_log, dt_bias, has_lower_bound, lower_bound, beta, b_gate,

@@ -897,7 +897,7 @@ static hipError_t fwd_h_segmented_dispatch(const void* k, const void* w, const v
   if (K != KD || V != VD || chunk != C || T <= 0 || T % C || B <= 0 || H <= 0) return hipErrorInvalidValue;
   if (!k || !w || !u || !h || !v_new || (!workspace && (!SPLIT || segments > 1))) return hipErrorInvalidValue;
   if (gate_mode != RG_NONE && !g) return hipErrorInvalidValue;
-  if (segments < 1 || segments > T / C) return hipErrorInvalidValue;
+  if (segments < 1 || segments > T / C || !aligned16(workspace)) return hipErrorInvalidValue;
   const int HQ = k_heads > 0 ? k_heads : H;
   if (H % HQ) return hipErrorInvalidValue;
   const int bv = value_block > 0 ? value_block : fwd_default_bv(B * segments, H);

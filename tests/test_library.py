@@ -319,6 +319,32 @@ def test_integration_guide_ctypes_lines_match_the_bindings():
     assert seen >= 10
 
 
+def test_misaligned_buffers_are_refused():
+    """The operands and workspaces that kernels touch in 16-byte pieces, refused on the host before any launch
+    (the other pointers are never followed)."""
+    from rewy_amd import _lib
+    lib, p = _lib.load(), 4096
+    none = [None] * 3
+
+    def prepare(operands, tail):      # fdr_fwd_prepare_scan's leading arguments: DeltaNet, fp32 beta
+        return [p, p, p, None, 0, 0, None, None, 0, 0.0, p, None, None, 0.0, 0, 0.0, *[None] * 8, operands, *tail]
+
+    def calls(operands, workspace, segments):
+        yield lib.fdr_fwd_scan_o(operands, 0, None, p, None, 0, *none[:2], 1, 128, 1, 128, 128, 64, 1.0, 0, segments,
+                                 workspace, None)
+        tail = [None, p, None, 0, *none, 1, 128, 1, 1, 1, 128, 128, 64, 1.0, 0, segments, workspace, None]
+        yield lib.fdr_forward_scan(*prepare(operands, tail))
+        yield lib.fdr_forward_scan_split(*prepare(operands, tail))
+    for off in (1, 4, 8, 15):
+        assert lib.fdr_fwd_prepare_scan(*prepare(p + off, [None, None, 1, 128, 1, 1, 128, 128, 64, 1.0, None])) == \
+            HIP_ERROR_INVALID_VALUE
+        for st in [*calls(p + off, None, 1), *calls(p, p + off, 2)]:
+            assert st == HIP_ERROR_INVALID_VALUE
+        for f in (lib.fdr_fwd_h_segmented, lib.fdr_fwd_h_split):
+            assert f(p, p, p, None, 0, None, p, p, None, 0, 1, 128, 1, 1, 128, 128, 64, 2, 0, p + off, None) == \
+                HIP_ERROR_INVALID_VALUE
+
+
 def test_varlen_takes_what_as_tensor_takes():
     """Lists, tuples, arrays and lists of scalar tensors; not text, wrong shapes or falling offsets.  Not on a
     default device either."""
