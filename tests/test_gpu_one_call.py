@@ -32,6 +32,28 @@ def test_forward_call(op, lens):
         assert (a is None and r is None) or torch.equal(a, r)
 
 
+def test_forward_call_takes_the_tile_it_is_given(monkeypatch):
+    """value_block on a packed batch is the caller's, the rule's only without one; other widths are refused."""
+    from rewy_amd import ops
+    xs, _ = make_inputs("kda", 1, 130, 2, seed=71)
+    xs = {n: x.cuda() for n, x in xs.items() if n != "initial_state"}
+    vl = ops.Varlen([0, 65, 130], xs["q"].device)
+    run = lambda **kw: ops.forward_scan(xs["q"], xs["k"], xs["v"], xs["g"], 2, beta=xs["beta"], **kw)  # noqa: E731
+    asked = []
+    real = ops.packed_tile
+    monkeypatch.setattr(ops, "packed_tile", lambda *a: (asked.append(a), real(*a))[1])
+    want = run(varlen=vl)[0]
+    assert len(asked) == 1
+    for vb in (16, 32, 64):
+        assert torch.equal(run(varlen=vl, value_block=vb)[0], want)
+    assert len(asked) == 1
+    xd = {n: x[:, :128].contiguous() for n, x in xs.items()}
+    for x, batch in ((xs, vl), (xd, None)):
+        for vb in (8, 48, -16):
+            with pytest.raises(ValueError):
+                ops.forward_scan(x["q"], x["k"], x["v"], x["g"], 2, beta=x["beta"], varlen=batch, value_block=vb)
+
+
 @pytest.mark.parametrize("op", ["delta", "gdn"])
 @pytest.mark.parametrize("vf,states", [(False, True), (True, True), (False, False)])
 def test_affine_backward_call(op, vf, states, monkeypatch):
