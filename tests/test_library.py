@@ -379,6 +379,20 @@ def test_packed_tile_rules():
     assert ops.packed_pair(vl(*[64] * 16), 16) is None
 
 
+def test_forward_scan_form_rules():
+    """fwd_form: segments on long rows up to the most heads at which three of them fit, the affine-step form
+    on short rows of very few heads, else direct."""
+    from rewy_amd import ops
+    for N, H, NT, form in ((1, 40, 256, "segmented"), (1, 41, 256, "direct"), (1, 43, 1024, "direct"),
+                           (1, 47, 4096, "direct"), (2, 20, 1024, "segmented"), (1, 32, 255, "direct"),
+                           (1, 31, 96, "segmented"), (1, 4, 127, "affine"), (1, 4, 128, "segmented"),
+                           (1, 1, 512, "segmented"), (1, 1, 511, "affine"), (1, 8, 7, "direct"), (1, 9, 64, "direct")):
+        assert ops.fwd_form(N, H, NT) == form, (N, H, NT)
+    for H in range(1, 65):
+        if ops.fwd_form(1, H, 4096) == "segmented":
+            assert ops.segments_for(1, H, 4096) >= 3
+
+
 def test_scan_segment_rules():
     """scan_segments: one scan with many heads or short rows; else segments of at least 16 chunks, at most 16,
     whose 64-wide tiles (two a head) give at most a work-group a CU."""
