@@ -385,8 +385,10 @@ def test_forward_scan_form_rules():
     from rewy_amd import ops
     for N, H, NT, form in ((1, 40, 256, "segmented"), (1, 41, 256, "direct"), (1, 43, 1024, "direct"),
                            (1, 47, 4096, "direct"), (2, 20, 1024, "segmented"), (1, 32, 255, "direct"),
-                           (1, 31, 96, "segmented"), (1, 4, 127, "affine"), (1, 4, 128, "segmented"),
-                           (1, 1, 512, "segmented"), (1, 1, 511, "affine"), (1, 8, 7, "direct"), (1, 9, 64, "direct")):
+                           (1, 16, 96, "segmented"), (1, 16, 95, "direct"), (1, 17, 127, "direct"),
+                           (1, 31, 128, "segmented"), (1, 9, 47, "direct"), (1, 9, 48, "affine"),
+                           (3, 4, 95, "affine"), (1, 13, 95, "direct"), (1, 4, 127, "affine"), (1, 4, 128, "segmented"),
+                           (1, 1, 512, "segmented"), (1, 1, 511, "affine"), (1, 8, 7, "direct"), (1, 8, 8, "affine")):
         assert ops.fwd_form(N, H, NT) == form, (N, H, NT)
     for H in range(1, 65):
         if ops.fwd_form(1, H, 4096) == "segmented":
