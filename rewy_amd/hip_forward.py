@@ -34,13 +34,22 @@ def _as(x, dtype):
     return x.to(dtype).contiguous()
 
 
-def _states_form(N, H, HQ, NT):
+STATES_MIN_CHUNKS = 64
+
+
+def _states_form(N, H, HQ, NT, keep, act):
     """The state scan's form where a forward that keeps no states is still faster with the scan's own
-    pass and ``fwd_o``, or None: the affine-step form on the short rows of one to four heads that
-    ``ops.scan_segments`` does not split.  Whole forward, KDA (graph replay, us), affine-step / the scan that
-    forms the output: H=4 64 chunks 86 / 97, H=2 64 chunks 82 / 95 (90 in segments), 32 chunks 62 / 64,
-    H=8 64 chunks 106 / 103, H=4 96 chunks 123 / 134 (111 in segments)."""
-    return "affine" if HQ == H and N * H <= 4 and 32 < NT and ops.scan_segments(N, H, NT) == 1 else None
+    pass and ``fwd_o``, or None: the affine-step form, for inference (``keep`` None) without activations
+    (``act``) on the short rows of one to four heads that ``ops.scan_segments`` does not split.  The form's
+    several library calls are host time, its steps shorter.  Whole eager calls (us, affine-step / the scan that
+    forms the output): DeltaNet H=4 48 chunks 74 / 65, 64 chunks 74 / 81, 95 chunks 99 / 114; KDA H=1 48 chunks
+    80 / 75, 64 chunks 80 / 94, 95 chunks 96 / 130; with raw q, k and beta KDA H=2 64 chunks 112 / 89, 95 chunks
+    113 / 121 (waited for after each call 193 / 165); forward and backward KDA H=2 64 chunks 365 / 312, 95 chunks
+    368 / 318, DeltaNet H=4 95 chunks 269 / 241."""
+    if keep is None and not act and HQ == H and N * H <= 4 and NT >= STATES_MIN_CHUNKS \
+            and ops.scan_segments(N, H, NT) == 1:
+        return "affine"
+    return None
 
 
 def chunk_forward_hip(op, q, k, v, g=None, beta=None, b=None, w=None, initial_state=None, scale=None,
@@ -79,7 +88,7 @@ def chunk_forward_hip(op, q, k, v, g=None, beta=None, b=None, w=None, initial_st
     form = "auto" if varlen is None else "direct"
     split = varlen is None and ops.split_pays(N, H, T // ops.CHUNK)
     if keep != "all" and varlen is None:
-        form = _states_form(N, H, HQ, T // ops.CHUNK)
+        form = _states_form(N, H, HQ, T // ops.CHUNK, keep, norm or beta_act)
     if keep != "all" and (varlen is not None or form is None):
         o, final, saved = ops.forward_scan(q, k, v, g, gm, beta=beta, b=b, w=w, scale=scale, h0=h0,
                                            want_final=output_final_state, state_v_first=state_v_first, varlen=varlen,

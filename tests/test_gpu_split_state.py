@@ -55,7 +55,8 @@ def test_split_forms_agree(op, B, NT, H, groups, vf, h0):
 
 @pytest.mark.parametrize("op,T,H,keep", [
     ("delta", 512, 2, None), ("gdn", 512, 2, "matrices"), ("kda", 512, 2, None), ("gdn2", 1024, 3, "matrices"),
-    ("kda", 1024, 16, "all"), ("gdn2", 576, 9, "all"), ("delta", 64 * 96, 2, None), ("kda", 64 * 128, 4, "all")])
+    ("kda", 1024, 16, "all"), ("gdn2", 576, 9, "all"), ("gdn", 64 * 64, 4, None), ("delta", 64 * 96, 2, None),
+    ("kda", 64 * 128, 4, "all")])
 def test_final_state_is_as_precise_as_the_affine_step_form(op, T, H, keep):
     from rewy_amd import ops
     from rewy_amd.hip_forward import chunk_forward_hip

@@ -379,6 +379,16 @@ def test_packed_tile_rules():
     assert ops.packed_pair(vl(*[64] * 16), 16) is None
 
 
+def test_stateless_forward_form_rule():
+    """_states_form: the affine-step form for plain inference on 64 to 95 chunks of one to four heads only."""
+    from rewy_amd.hip_forward import _states_form
+    assert _states_form(1, 4, 4, 64, None, False) == _states_form(2, 2, 2, 95, None, None) == "affine"
+    for N, H, HQ, NT, keep, act in ((1, 4, 4, 63, None, False), (1, 4, 4, 96, None, False), (1, 5, 5, 64, None, False),
+                                    (1, 4, 2, 64, None, False), (1, 4, 4, 64, "matrices", False),
+                                    (1, 4, 4, 64, None, True), (1, 1, 1, 64, None, 2.0)):
+        assert _states_form(N, H, HQ, NT, keep, act) is None
+
+
 def test_forward_scan_form_rules():
     """fwd_form: segments on long rows up to the most heads at which three of them fit, the affine-step form
     on short rows of very few heads, else direct."""
