@@ -8,8 +8,7 @@ and returns the same (o, final_state, saved) as ``rewy_amd.forward.chunk_forward
 
   1. ``fdr_fwd_prepare_wu`` -- gc (log2 chunk-local cumsum), Aqk, Akk = (I + M)^-1, w, u
      (and kg, qg for vector gates);
-  2. ``fdr_fwd_h``          -- per-chunk states h, v_new and the final state
-     (or ``fdr_fwd_prepare`` and w / u in the scan, ``fdr_fwd_h_wy``, where that pays);
+  2. ``fdr_fwd_h``          -- per-chunk states h, v_new and the final state;
   3. ``fdr_fwd_o``          -- o = scale (q 2^gc) h + Aqk v_new.
 
 Where no backward reads the states (recompute policy, inference) two launches instead:
@@ -53,14 +52,16 @@ def _states_form(N, H, HQ, NT, keep, act):
 
 
 def chunk_forward_hip(op, q, k, v, g=None, beta=None, b=None, w=None, initial_state=None, scale=None,
-                      output_final_state=False, varlen=None, state_v_first=False, fuse_scan=None, want_qg=True,
+                      output_final_state=False, varlen=None, state_v_first=False, fuse_scan=False, want_qg=True,
                       gate=None, keep="all", norm=False, beta_act=None):
     """``varlen`` (an ``ops.Varlen``): B = 1 holds sequences packed along T, starting
     anywhere (FLA's cu_seqlens); initial / final states are per sequence, and every stage
     takes the batch's chunk map (a sequence's last chunk may be partial).  ``state_v_first``:
     initial / final states are [N,H,V,K] (read and written so by ``fwd_h``); the saved
-    per-chunk h stays [B,NT,H,K,V].  ``fuse_scan``: w / u in the scan (``fdr_fwd_h_wy``,
-    the same bits, u not materialized: saved ``u`` is None) -- by default where that pays.
+    per-chunk h stays [B,NT,H,K,V].  ``fuse_scan`` (``keep`` "all"): w / u in the scan (``fdr_fwd_h_wy``,
+    the same bits, u not materialized: saved ``u`` is None).  No operator asks for it: step 1 forms w / u at a
+    third of ``fdr_prepare_wu``'s cost, which leaves the sweep nothing for a vector gate (KDA B=8 T=4096 H=16
+    738 us, with the sweep 827), and the other families' forward keeps no states.
     ``gate`` (KDA) = (lower_bound, A_log, dt_bias): g is the raw gate, activated inside step 1.
     ``want_qg=False``: saved ``qg`` is None (only a backward that recomputes nothing reads it).
 
@@ -72,6 +73,8 @@ def chunk_forward_hip(op, q, k, v, g=None, beta=None, b=None, w=None, initial_st
     s * sigmoid(beta) -- on load in step 1 where the states stay on the chip, else by passes of their
     own.  Saved then also hold what the backward reads: the normalised q, k with their rows' 1 / norm
     rq, rk, and the activated beta."""
+    if fuse_scan and keep != "all":
+        raise ValueError('fuse_scan: the sweep keeps the states (keep="all")')
     B, T, HQ, K = q.shape
     scale = K ** -0.5 if scale is None else scale
     gm = GATE_MODE[op]
@@ -103,11 +106,6 @@ def chunk_forward_hip(op, q, k, v, g=None, beta=None, b=None, w=None, initial_st
     if beta_act:
         from .gates import beta_sigmoid
         beta = beta_sigmoid(beta, beta_act, native=True)
-    if fuse_scan is None:
-        # fdr_fwd_prepare_wu forms w / u at a third of prepare_wu's cost, so the sweep pays only for the
-        # scalar / no-gate families at 64-wide tiles (forward, us, pair / sweep: GDN B=8 T=4096 H=16
-        # 563 / 548, B=4 T=2048 H=16 170 / 180; KDA B=8 T=4096 H=16 738 / 827)
-        fuse_scan = not vec and ops.default_tile(N, H) == 64 and ops.fwd_h_wy_pays(N, H, gm, varlen)
     if fuse_scan:
         if gate is not None:
             from .gates import kda_gate

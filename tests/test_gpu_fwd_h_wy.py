@@ -157,3 +157,13 @@ def test_hip_forward_fused_scan_equals_the_pair(op):
     for n in ("w", "qg", "kg", "h", "v_new"):
         if s0[n] is not None:
             assert torch.equal(s1[n], s0[n]), n
+
+
+def test_hip_forward_fused_scan_is_refused_without_states():
+    """A forward that keeps no states cannot run the sweep: an error, not another form."""
+    from rewy_amd.hip_forward import chunk_forward_hip
+    xs, _ = make_inputs("gdn", 1, 128, 2, seed=67)
+    xs = {n: x.cuda() for n, x in xs.items()}
+    for keep in ("matrices", None):
+        with pytest.raises(ValueError, match="fuse_scan"):
+            chunk_forward_hip("gdn", xs["q"], xs["k"], xs["v"], g=xs["g"], beta=xs["beta"], keep=keep, fuse_scan=True)
