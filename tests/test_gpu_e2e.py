@@ -210,3 +210,52 @@ def test_optimized_varlen_and_v_first_match_original(op):
         with fdr.use_backend("optimized", ops=(op,)):
             with pytest.raises(RuntimeError, match="grouped heads or unequal q/k/v shapes"):
                 getattr(fdr, OPNAME[op])(**args)
+
+
+@pytest.mark.parametrize("op,groups,kw", [
+    ("gdn", 2, {}), ("gdn", 1, {}), ("kda", 2, dict(disable_recompute=False)), ("kda", 2, dict(disable_recompute=True)),
+    ("kda", 1, dict(disable_recompute=True)), ("gdn2", 1, dict(disable_recompute=False)), ("delta", 2, {})])
+@pytest.mark.parametrize("lens", [(1, 65, 62), (128,)])
+def test_raw_inputs_in_packed_grouped_batches(op, groups, kw, lens):
+    """use_qk_l2norm_in_kernel and use_beta_sigmoid_in_kernel over packed partial chunks and grouped value heads:
+    the output, the final states and every raw input's gradient against the token recurrence in fp64, each
+    sequence by itself.  q and k rows of different lengths, so that a swapped or missing norm shows."""
+    import rewy_amd as fdr
+    print(f"\n[e2e-raw] op={op} groups={groups} kw={kw} lens={lens}", flush=True)
+    T, H, N = sum(lens), 4, len(lens)
+    xs, dO = make_inputs(op, 1, T, H, seed=37)
+    gen = torch.Generator().manual_seed(38)
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    xs["initial_state"] = rnd(N, H, 128, 128) * 0.02
+    for n, s in (("q", 3.0), ("k", 0.3)):
+        xs[n] = (rnd(1, T, H // groups, 128) * s * (0.5 + torch.rand(1, T, H // groups, 1, generator=gen))).bfloat16()
+    act = op in ("gdn", "kda")
+    if act:
+        xs["beta"] = rnd(1, T, H)
+        kw = dict(kw, use_beta_sigmoid_in_kernel=True)
+    dht = rnd(N, H, 128, 128) * 0.1
+    dev = torch.device("cuda")
+    xg = {n: x.to(dev).requires_grad_() for n, x in xs.items()}
+    cu = torch.tensor([0, *lens]).cumsum(0)
+    with fdr.use_backend("optimized"):
+        o, ht = getattr(fdr, OPNAME[op])(**xg, output_final_state=True, use_qk_l2norm_in_kernel=True,
+                                         cu_seqlens=cu.to(dev), **kw)
+    got = dict(zip(xs, torch.autograd.grad((o, ht), tuple(xg.values()), (dO.to(dev), dht.to(dev)))))
+    x64 = {n: x.double().requires_grad_() for n, x in xs.items()}
+    ys = dict(x64)
+    for n in ("q", "k"):
+        y = x64[n] * torch.rsqrt((x64[n] ** 2).sum(-1, keepdim=True) + 1e-6)
+        ys[n] = y.repeat_interleave(groups, dim=2)
+    if act:
+        ys["beta"] = torch.sigmoid(x64["beta"])
+    out = [O.torch_token_recurrence(op, {n: y[i:i + 1] if n == "initial_state" else y[:, a:e] for n, y in ys.items()})
+           for i, (a, e) in enumerate(zip(cu.tolist(), cu.tolist()[1:]))]
+    want_o, want_ht = torch.cat([x[0] for x in out], 1), torch.cat([x[1] for x in out])
+    want = dict(zip(xs, torch.autograd.grad((want_o, want_ht), tuple(x64.values()), (dO.double(), dht.double()))))
+    n = lambda x: x.detach().double().cpu().numpy()  # noqa: E731
+    for a, r in ((o, want_o), (ht, want_ht)):
+        e = O.error(n(r), n(a), O.limit_for("dq"))
+        assert e["passed"], e
+    for name in xs:
+        e = O.error(n(want[name]), n(got[name]), O.limit_for(GRAD[name]))
+        assert e["passed"], (name, e)
