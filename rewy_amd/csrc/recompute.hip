@@ -514,7 +514,8 @@ __global__ __launch_bounds__(512) void fwd_h_kernel(
 // they share every staged operand; nothing per chunk is stored.  The per-chunk arithmetic is
 // fwd_h_kernel's.  A scan of 1024 chunks at B*H = 16 is bound by its step chain with most CUs idle:
 // 1393 us direct and 1773 affine-step, against 624 in all for the maps, the chain and eight segments
-// of 128 (4 segments 965, 16 664).  P goes to pbuf [rows*segs, H, K, K], Q to qbuf [rows*segs, H, K, V].
+// of 128 (4 segments 965, 16 664), hi + lo 5-9 % more (this kernel 287 -> 342: Q's rest is read by every
+// wave, and LDS fills the step).  P goes to pbuf [rows*segs, H, K, K], Q to qbuf [rows*segs, H, K, V].
 template <bool SPLIT>
 struct FwdXferSmem {
   static constexpr int LDK = KD + 8;
