@@ -21,7 +21,7 @@ BUILD = HERE / "_build"
 ARCH = "gfx950"
 FLAGS = [
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
-    # packed fp32 ops off: some of their forms have given wrong results on this pool
+    # packed fp32 ops off: some of their forms have given wrong results on this hardware
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I", str(HERE.parent / "include"),
 ]

@@ -1,4 +1,4 @@
-"""Seeded synthetic inputs shared by the tests (BASELINE.json distributions)."""
+"""Seeded synthetic inputs shared by the tests (the benchmark's distributions)."""
 import torch
 import torch.nn.functional as F
 
@@ -23,7 +23,7 @@ def make_inputs(op, B, T, H, K=128, seed=0, gate="default", h0=True, beta_zero_e
     elif op in ("kda", "gdn2"):
         if gate == "wide":
             xs["g"] = F.logsigmoid(torch.randn(shape, generator=g_) * 3 - 4)
-        elif gate == "mild":      # long-memory gates (BASELINE.json's kda_long draw)
+        elif gate == "mild":      # long-memory gates (the long-context workload's draw)
             xs["g"] = F.logsigmoid(torch.randn(shape, generator=g_) * 0.3 + 3)
         else:
             xs["g"] = F.logsigmoid(torch.randn(shape, generator=g_)).clamp_min(-5)

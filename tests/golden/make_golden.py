@@ -1,6 +1,6 @@
 """Write the per-family golden vectors tests/golden/family_<op>.npz.
 
-Inputs are the seeded BASELINE.json-style tensors of tests/_inputs.py at
+Inputs are the seeded benchmark-style tensors of tests/_inputs.py at
 B=1, T=128 (two chunks), H=1, K=V=128 with beta zero on every 5th token
 (scalar-beta families); bf16 tensors are stored as their uint16 bit patterns.
 Outputs are the fp64 oracle's gradients (rounded to fp32) of

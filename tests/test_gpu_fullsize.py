@@ -1,4 +1,4 @@
-"""The BASELINE.json workloads at their full sizes: the optimized path (HIP
+"""The benchmark's workloads at their full sizes: the optimized path (HIP
 forward + HIP backward) against the original-formulation backend (PyTorch ops,
 fp32) on the same inputs, through the public autograd operators, at the
 reference's acceptance tolerances (validation.py:40-45: rel-L2 <= 0.008 for

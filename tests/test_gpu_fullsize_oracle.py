@@ -1,4 +1,4 @@
-"""The BASELINE.json workloads at their full sizes against the fp64 oracle, head by head.
+"""The benchmark's workloads at their full sizes against the fp64 oracle, head by head.
 
 Every (batch row, head) pair of the chunked delta rule is independent end to end, so the
 gradients the optimized path (HIP forward + HIP backward, through the public autograd

@@ -5,7 +5,7 @@ against the residual kernel on the same inputs.
 The oracle's stage function computes the chunk-stage gradients from the closed form
 (pinned by complex step against the token recurrence), independently of which product
 list forms them, so both formulations must meet it; tolerances as for the residual kernel
-(rel-L2 1e-2 for bf16 outputs, 5e-3 for fp32).  Cases: the BASELINE gate distribution, rows
+(rel-L2 1e-2 for bf16 outputs, 5e-3 for fp32).  Cases: the benchmark's gate distribution, rows
 with beta = 0 (dbeta's direct VJP is the original's rule on every row), wide gate spans
 (the pairwise intra diagonal), several chunks and heads.
 """
